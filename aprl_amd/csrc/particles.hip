@@ -29,7 +29,7 @@ struct GArgs {
   const double* b[3];      // B^(n+1/2)
   int ne[3][3], nb[3][3];  // (nx, ny, nz) of E (= J) and B components
   int nx, ny, nz;          // cells
-  double o[3], h[3], ih[3];  // origin, spacing, 1 / spacing
+  double o[3], h[3];
   double negS;             // (-1*dt)/eps0, applyCurrentSource(-1)
   int smoothX;
   // the Picard stop word: a trial's kernels return at once when it is set
@@ -55,7 +55,7 @@ struct PArgs {
   const double* beta;  // held speed of held entries
   const unsigned* tileOf;         // sorted tile key of each entry
   unsigned long long* tileBound;  // per tile: largest particle current bound
-  double scaleInv;   // 1 / (dx dy dz dt)
+  double scaleDen;   // dx*dy*dz*dt
   int n;
 };
 
@@ -102,23 +102,26 @@ __device__ Clip clipOrbit(const GArgs& G, const double begin[3], const double en
 
 // The chord begin -> end in cells from the grid's origin, clipped to the grid
 // (clipOpenOrbit): start x, displacement v, kept fraction. A chord that lies
-// in the grid needs none of the clip's divisions.
+// in the grid needs none of the clip's divisions. x is the quotient that
+// names the start's tile (kTileKeys): a product with 1 / h differs from it by
+// a rounding, and a chord that starts on a tile's face and moves a whole cell
+// would then leave its tile's box.
 __device__ __forceinline__ bool chordInGrid(const GArgs& G, const double begin[3], const double end[3], double x[3],
                                             double v[3], double& kept, unsigned& err) {
   const int size[3] = {G.nx, G.ny, G.nz};
   bool inside = true;
   for (int a = 0; a < 3; ++a) {
-    x[a] = (begin[a] - G.o[a]) * G.ih[a];
-    v[a] = (end[a] - begin[a]) * G.ih[a];
-    const double last = (end[a] - G.o[a]) * G.ih[a], n = size[a];
+    x[a] = (begin[a] - G.o[a]) / G.h[a];
+    v[a] = (end[a] - begin[a]) / G.h[a];
+    const double last = x[a] + v[a], n = size[a];
     inside = inside && x[a] >= 0. && x[a] <= n && last >= 0. && last <= n;
   }
   kept = 1.;
   if (inside) return true;
   const Clip path = clipOrbit(G, begin, end, err);
   for (int a = 0; a < 3; ++a) {
-    x[a] = (path.b[a] - G.o[a]) * G.ih[a];
-    v[a] = (path.e[a] - path.b[a]) * G.ih[a];
+    x[a] = (path.b[a] - G.o[a]) / G.h[a];
+    v[a] = (path.e[a] - path.b[a]) / G.h[a];
   }
   kept = path.last - path.first;
   return path.valid;
@@ -598,9 +601,9 @@ kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin,
       for (int d = 0; d < 3; ++d) {
         const double s0 = leg ? xk[d] : xa[d], s1 = last ? xb[d] : xk[d];
         // scale_a = q * (x1_a - x0_a) / (dx dy dz dt), eb_deposition.cpp:41-51
-        scale[d] = q * (s1 - s0) * P.scaleInv;
-        x[d] = (s0 - G.o[d]) * G.ih[d];
-        v[d] = (s1 - s0) * G.ih[d];
+        scale[d] = q * (s1 - s0) / P.scaleDen;
+        x[d] = (s0 - G.o[d]) / G.h[d];
+        v[d] = (s1 - s0) / G.h[d];
       }
       const int count = orbitCuts(x, v, cuts, err);
       const double f1 = last ? t1 : 1.0, f2 = last ? t2 : 1.0, fw = last ? wCarrier : 0.0;
@@ -688,7 +691,6 @@ static GArgs gatherArgs(const CouplingState& C, const FieldState& F, const doubl
   G.ny = static_cast<int>(F.g.ny);
   G.nz = static_cast<int>(F.g.nz);
   G.h[0] = F.g.dx; G.h[1] = F.g.dy; G.h[2] = F.g.dz;
-  for (int a = 0; a < 3; ++a) G.ih[a] = 1.0 / G.h[a];
   G.negS = -1.0 * F.g.dt / kEps0;
   G.smoothX = C.smoothX ? 1 : 0;
   return G;
@@ -1364,7 +1366,7 @@ void plainStepBegin(CouplingState& C, ParticleStore& P, const double origin[3], 
 
   X.S = stepArgsFor(C, F.g, F.hasCpml ? &F.cpml : nullptr, F.window, origin, time, substeps);
   X.A = particleArgs(P);
-  X.A.scaleInv = 1.0 / (F.g.dx * F.g.dy * F.g.dz * F.g.dt);
+  X.A.scaleDen = F.g.dx * F.g.dy * F.g.dz * F.g.dt;
   X.A.tileOf = P.keySorted.get();
   X.A.tileBound = C.tileBound.get();
   X.G = gatherArgs(C, F, origin);
