@@ -533,7 +533,7 @@ __global__ void __launch_bounds__(128) kPush(PArgs P, GArgs G, StepArgs S, unsig
 template <int SHAPE>
 __global__ void __launch_bounds__(kChunk) __attribute__((amdgpu_waves_per_eu(SHAPE == kShapeQuintic ? 2 : 3)))
 kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin, const int* tileEnd,
-         const unsigned long long* tileScan, int ntx, int nty, long long* partial, int* tileShift, unsigned* errOut) {
+         const unsigned long long* tileScan, int ntx, int nty, TileBoxes T, int* tileShift, unsigned* errOut) {
   if (G.stop && *G.stop) return;
   using W = RawBox<SHAPE>;
   constexpr int N = rawNodes<SHAPE>();
@@ -623,7 +623,7 @@ kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin,
     }
   }
   __syncthreads();
-  flushRawBox<SHAPE>(acc, box, G.ne, partial, tileScan, tile);
+  flushRawBox<SHAPE>(acc, box, G.ne, T, tileScan, tile);
   if (err) atomicOr(errOut, err);
 }
 
@@ -646,11 +646,11 @@ kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin,
 template <int SHAPE>
 __global__ void __launch_bounds__(256) kReduceCurrent(double* jx, double* jy, double* jz, GArgs G, const int* active,
                                                       const unsigned long long* tileScan, const int* tileShift,
-                                                      long long* partial, int ntx, int nty, int ntz, int writeJ) {
+                                                      TileBoxes T, int ntx, int nty, int ntz, int writeJ) {
   if (G.stop && *G.stop) return;
   const int tile = active[xcdContiguous(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   reduceOwnedTile<SHAPE>(
-      G.ne, tile, tileScan, tileShift, partial, ntx, nty, ntz,
+      G.ne, tile, tileScan, tileShift, T, ntx, nty, ntz,
       [&](int i, int j, int k, const bool has[3], const double sum[3]) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -1013,15 +1013,21 @@ void reduceChunkStats(hipStream_t st, const double* in, int chunks, double* out)
   launchCheck("chunk stats");
 }
 
-void reserveStepBuffers(CouplingState& C, std::size_t partialNeed, unsigned nChunks, hipStream_t st) {
-  if (partialNeed > C.partial.size()) {
-    // the larger tiles' boxes must start at zero; the reduction keeps them so
-    const std::size_t n = partialNeed + partialNeed / 2;
-    C.partial.resize(n);
-    hipCheck(hipMemsetAsync(C.partial.get(), 0, n * sizeof(long long), st), "hipMemsetAsync");
+TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, unsigned nChunks, unsigned occupied,
+                             hipStream_t st) {
+  const std::size_t extra = nChunks - occupied, added = std::min<std::size_t>(extra, occupied);
+  if (added > C.addedBoxes || occupied > C.storedBoxes) {
+    const std::size_t zeros = added > C.addedBoxes ? added + added / 2 : C.addedBoxes;
+    const std::size_t others = occupied > C.storedBoxes ? occupied + occupied / 2 : C.storedBoxes;
+    C.addedBoxes = C.storedBoxes = 0;  // none, should the allocation fail
+    C.boxes.resize(boxWords * (zeros + others));
+    if (zeros) hipCheck(hipMemsetAsync(C.boxes.get(), 0, boxWords * zeros * sizeof(long long), st), "hipMemsetAsync");
+    C.addedBoxes = zeros;
+    C.storedBoxes = others;
   }
   const std::size_t blocks = 4 * static_cast<std::size_t>(std::max(1u, nChunks));
   if (C.reduceBlocks.size() < blocks) C.reduceBlocks.resize(blocks + blocks / 2);
+  return TileBoxes{C.boxes.get(), static_cast<int>(C.addedBoxes), extra <= occupied ? 1 : 0};
 }
 
 void reserveCouplingWords(CouplingState& C, hipStream_t st) {
@@ -1183,6 +1189,7 @@ struct PlainStepContext {
   unsigned commitAfter = 0;    // trials ahead of the gated E commit (0: none enqueued)
   bool quintic = false;
   double origin[3] = {0.0, 0.0, 0.0};
+  TileBoxes boxes{};
   PArgs A{};
   GArgs G{};
   StepArgs S{};
@@ -1233,11 +1240,11 @@ void enqueueTrials(CouplingState& C, PlainStepContext& X, unsigned first, unsign
         if (quintic)
           kDeposit<kShapeQuintic><<<nChunks, kChunk, 0, st>>>(
               A, G, S, C.chunks.get(), C.tileBegin.get(), C.tileEnd.get(), C.tileScan.get(), ntx, nty,
-              C.partial.get(), C.tileShift.get(), errT);
+              X.boxes, C.tileShift.get(), errT);
         else
           kDeposit<kShapeBinomial3X><<<nChunks, kChunk, 0, st>>>(
               A, G, S, C.chunks.get(), C.tileBegin.get(), C.tileEnd.get(), C.tileScan.get(), ntx, nty,
-              C.partial.get(), C.tileShift.get(), errT);
+              X.boxes, C.tileShift.get(), errT);
         launchCheck("deposit");
       }
       {
@@ -1247,12 +1254,12 @@ void enqueueTrials(CouplingState& C, PlainStepContext& X, unsigned first, unsign
         if (quintic)
           kReduceCurrent<kShapeQuintic><<<nActive, 256, 0, st>>>(F.base(6), F.base(7), F.base(8), G,
                                                                  C.activeTiles.get(), C.tileScan.get(),
-                                                                 C.tileShift.get(), C.partial.get(), ntx, nty, ntz,
+                                                                 C.tileShift.get(), X.boxes, ntx, nty, ntz,
                                                                  writeJ);
         else
           kReduceCurrent<kShapeBinomial3X><<<nActive, 256, 0, st>>>(F.base(6), F.base(7), F.base(8), G,
                                                                     C.activeTiles.get(), C.tileScan.get(),
-                                                                    C.tileShift.get(), C.partial.get(), ntx, nty,
+                                                                    C.tileShift.get(), X.boxes, ntx, nty,
                                                                     ntz, writeJ);
         launchCheck("reduce current");
       }
@@ -1361,8 +1368,7 @@ void plainStepBegin(CouplingState& C, ParticleStore& P, const double origin[3], 
   }
   const bool quintic = C.shape == kShapeQuintic;
   const int boxN = quintic ? boxNodes<kShapeQuintic>() : boxNodes<kShapeBinomial3X>();
-  const std::size_t partialNeed = static_cast<std::size_t>(occupiedTiles) * 2 * 3 * boxN;
-  reserveStepBuffers(C, partialNeed, nChunks, st);
+  X.boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), nChunks, occupiedTiles, st);
 
   X.S = stepArgsFor(C, F.g, F.hasCpml ? &F.cpml : nullptr, F.window, origin, time, substeps);
   X.A = particleArgs(P);

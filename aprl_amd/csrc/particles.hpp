@@ -182,15 +182,16 @@ struct CouplingState {
   DeviceArray<unsigned long long> tileBound;
   // per tile (+1 entry for the scan totals): packed counts (chunks,
   // occupied, has an occupied neighbour; packTileCounts); the exclusive
-  // scan gives the first chunk, the partial slot and the active slot
+  // scan gives the first chunk, the occupied slot and the active slot
   DeviceArray<unsigned long long> tileCounts, tileScan;
   DeviceArray<int4> chunks;  // (tile, first particle, end particle, 0)
   std::size_t chunkCapacity = 0;
   DeviceArray<unsigned long long> tileSums;  // of tileCounts, per workgroup of kTileCounts
   DeviceArray<unsigned> keyActive;           // live active entries per workgroup of the key kernel
-  // per occupied tile (in tile order): 2 x 3 extended tile boxes of
-  // fixed-point current (coveringTiles)
-  DeviceArray<long long> partial;
+  // fixed-point current of the tiles, 3 components of an extended tile box
+  // each (TileBoxes), and the capacities of its two parts in boxes
+  DeviceArray<long long> boxes;
+  std::size_t addedBoxes = 0, storedBoxes = 0;
   DeviceArray<double> reduceBlocks, reduceOut;
   DeviceArray<unsigned> error;
   // cumulative boundary counters and their per-block partials
@@ -363,11 +364,23 @@ void appendParticles(ParticleStore& P, std::size_t k, const double* x3, const do
 // Error words and boundary counters of a coupling (allocated and cleared
 // once).
 void reserveCouplingWords(CouplingState& C, hipStream_t st);
-// The step's tile partials (zeroed) and residual block slots, grown with
-// half again as much headroom: a bunch that spreads over new tiles raises
-// the need a little in many steps, and every reallocation frees device
-// memory, which waits for the device.
-void reserveStepBuffers(CouplingState& C, std::size_t partialNeed, unsigned nChunks, hipStream_t st);
+// Fixed-point current boxes of the occupied tiles, in one array: the first
+// `added` boxes are those of tiles of several chunks, which add to zeros that
+// the reduction restores; the boxes behind them, by occupied slot, are those
+// of tiles of one chunk, which stores every node. A larger tile's box is its
+// first chunk less its occupied slot (it advances that difference by its
+// chunks beyond the first, so the difference is its own), or its occupied
+// slot where that makes fewer boxes (byChunk = 0).
+struct TileBoxes {
+  long long* at;
+  int added, byChunk;
+};
+// The step's tile boxes and residual block slots, grown with half again as
+// much headroom: a bunch that spreads over new tiles raises the need a little
+// in many steps, and every reallocation frees device memory, which waits for
+// the device. boxWords: 64-bit words of a tile's box.
+TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, unsigned nChunks, unsigned occupied,
+                             hipStream_t st);
 // Boundary-event commit after the converged trial: entry states and
 // weights, removed-entry count and the counters, skipped on the device when
 // the trial's error word carries no kEvtAny. R is the store's real type.

@@ -418,7 +418,7 @@ __global__ void __launch_bounds__(128) kPushSplit(PArgs32 P, StepArgs S, double 
 template <int SHAPE, bool LOOP>
 __global__ void __launch_bounds__(kChunk) __attribute__((amdgpu_waves_per_eu(SHAPE == kShapeQuintic ? 2 : 3)))
 kDepositSplit(PArgs32 P, GArgs32 G, StepArgs S, const int4* chunks, const int* tileBegin, const int* tileEnd,
-              const unsigned long long* tileScan, int ntx, int nty, long long* partial, int* tileShift,
+              const unsigned long long* tileScan, int ntx, int nty, TileBoxes T, int* tileShift,
               unsigned* errOut) {
   using W = RawBox<SHAPE>;
   constexpr int N = rawNodes<SHAPE>();
@@ -521,7 +521,7 @@ kDepositSplit(PArgs32 P, GArgs32 G, StepArgs S, const int4* chunks, const int* t
     if (p0 < ch.z) particle(p0);
   }
   __syncthreads();
-  flushRawBox<SHAPE>(acc, box, G.ne, partial, tileScan, tile);
+  flushRawBox<SHAPE>(acc, box, G.ne, T, tileScan, tile);
   if (err) atomicOr(errOut, err);
 }
 
@@ -533,11 +533,11 @@ kDepositSplit(PArgs32 P, GArgs32 G, StepArgs S, const int4* chunks, const int* t
 template <int SHAPE, bool J, bool ESUM>
 __global__ void __launch_bounds__(256) kReduceCurrentSplit(float* jx, float* jy, float* jz, GArgs32 G,
                                                            const int* active, const unsigned long long* tileScan,
-                                                           const int* tileShift, long long* partial, int ntx,
+                                                           const int* tileShift, TileBoxes T, int ntx,
                                                            int nty, int ntz) {
   const int tile = active[xcdContiguous(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   reduceOwnedTile<SHAPE>(
-      G.ne, tile, tileScan, tileShift, partial, ntx, nty, ntz,
+      G.ne, tile, tileScan, tileShift, T, ntx, nty, ntz,
       [&](int i, int j, int k, const bool has[3], const double sum[3]) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -1026,8 +1026,7 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
   }
   const bool quintic = C.shape == kShapeQuintic;
   const int boxN = quintic ? boxNodes<kShapeQuintic>() : boxNodes<kShapeBinomial3X>();
-  const std::size_t partialNeed = static_cast<std::size_t>(occupiedTiles) * 2 * 3 * boxN;
-  reserveStepBuffers(C, partialNeed, nChunks, st);
+  const TileBoxes boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), nChunks, occupiedTiles, st);
 
   const StepArgs& S = X.S;
   PArgs32 A = particleArgs32(P, F);
@@ -1067,7 +1066,7 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
       ScopedKernel sk(F.profiler, st, "deposit");
 #define APRL_DEPOSIT32(SH, L)                                                                                    \
   kDepositSplit<SH, L><<<nChunks, kChunk, 0, st>>>(A, G, S, C.chunks.get(), C.tileBegin.get(), C.tileEnd.get(),  \
-                                                   C.tileScan.get(), ntx, nty, C.partial.get(), C.tileShift.get(), errT)
+                                                   C.tileScan.get(), ntx, nty, boxes, C.tileShift.get(), errT)
       if (quintic) {
         if (loop) APRL_DEPOSIT32(kShapeQuintic, true);
         else APRL_DEPOSIT32(kShapeQuintic, false);
@@ -1086,7 +1085,7 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
       const bool writeJ = last || C.refCurrent;
 #define APRL_REDUCE32(SH, WJ, WE)                                                                                     \
   kReduceCurrentSplit<SH, WJ, WE><<<nActive, 256, 0, st>>>(j[0], j[1], j[2], G, C.activeTiles.get(), C.tileScan.get(), \
-                                                           C.tileShift.get(), C.partial.get(), ntx, nty, ntz)
+                                                           C.tileShift.get(), boxes, ntx, nty, ntz)
       if (quintic) {
         if (writeJ && esum) APRL_REDUCE32(kShapeQuintic, true, true);
         else if (writeJ) APRL_REDUCE32(kShapeQuintic, true, false);

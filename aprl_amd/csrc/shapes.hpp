@@ -375,19 +375,25 @@ __device__ __forceinline__ unsigned rawDepositMask(const TileBox<SHAPE>& box, co
   return mask;
 }
 
-// Fixed-point tile partials: per occupied tile two boxes of 3 components x
-// boxNodes<SHAPE>() 64-bit integers scaled by 2^shift (shift per tile), box
-// 2 f for a tile of one chunk (slot f), which stores every node and leaves
-// the box dirty, box 2 f + 1 for a larger tile, whose chunks add to zeros
-// and which the reduction clears again.
-//
+// Fixed-point tile boxes (TileBoxes): 3 components x boxNodes<SHAPE>() 64-bit
+// integers scaled by 2^shift (shift per tile). A tile's box from its scanned
+// counts; -1 for an unoccupied tile.
+__device__ __forceinline__ int tileBoxOf(const TileBoxes& T, unsigned long long scan, unsigned long long next) {
+  const int chunks = chunkField(next) - chunkField(scan);
+  if (chunks <= 0) return -1;
+  const int slot = occupiedField(scan);
+  if (chunks == 1) return T.added + slot;
+  return T.byChunk ? chunkField(scan) - slot : slot;
+}
+
 // The owner side's table of the covering tiles of tile (tx, ty, tz): threads
 // 0..9(2RZ+1)-1 fill, per neighbour offset (oz + RZ, oy + 1, ox + 1), the
-// box (-1: unoccupied) and the exponent from the tile scan. The caller
+// box (tileBoxOf) and the exponent from the tile scan. The caller
 // synchronizes before reading it.
 template <int SHAPE>
-__device__ __forceinline__ void coveringTiles(const unsigned long long* tileScan, const int* tileShift, int tx,
-                                              int ty, int tz, int ntx, int nty, int ntz, int* nbBox, int* nbShift) {
+__device__ __forceinline__ void coveringTiles(const TileBoxes& T, const unsigned long long* tileScan,
+                                              const int* tileShift, int tx, int ty, int tz, int ntx, int nty, int ntz,
+                                              int* nbBox, int* nbShift) {
   constexpr int RZ = Box<SHAPE>::RZ, NB = 9 * (2 * RZ + 1);
   if (threadIdx.x >= NB) return;
   const int nb = static_cast<int>(threadIdx.x);
@@ -395,12 +401,8 @@ __device__ __forceinline__ void coveringTiles(const unsigned long long* tileScan
   int box = -1, sh = 0;
   if (x >= 0 && x < ntx && y >= 0 && y < nty && z >= 0 && z < ntz) {
     const int s = (z * nty + y) * ntx + x;
-    const unsigned long long sc = tileScan[s];
-    const int chunks = chunkField(tileScan[s + 1]) - chunkField(sc);
-    if (chunks > 0) {
-      box = 2 * occupiedField(sc) + (chunks > 1 ? 1 : 0);
-      sh = tileShift[s];
-    }
+    box = tileBoxOf(T, tileScan[s], tileScan[s + 1]);
+    if (box >= 0) sh = tileShift[s];
   }
   nbBox[nb] = box;
   nbShift[nb] = sh;
@@ -414,7 +416,7 @@ __device__ __forceinline__ void coveringTiles(const unsigned long long* tileScan
 // box are cleared for the next deposit. has: whether the component owns the
 // node.
 template <int SHAPE>
-__device__ __forceinline__ void ownedNodeSums(long long* partial, const int* nbBox, const int* nbShift, int tx, int ty,
+__device__ __forceinline__ void ownedNodeSums(const TileBoxes& T, const int* nbBox, const int* nbShift, int tx, int ty,
                                               int tz, int i, int j, int k, const bool has[3], double sum[3]) {
   using B = Box<SHAPE>;
   constexpr int N = boxNodes<SHAPE>(), RZ = B::RZ;
@@ -434,14 +436,14 @@ __device__ __forceinline__ void ownedNodeSums(long long* partial, const int* nbB
         const int box = nbBox[nb];
         if (box < 0) continue;
         const int li = i - (x * kTileX - B::X0), lj = j - (y * kTileY - B::Y0), lk = k - (z * kTileZ - B::Z0);
-        long long* const at = partial + static_cast<size_t>(box) * 3 * N + (lk * B::NY + lj) * B::NX + li;
+        long long* const at = T.at + static_cast<size_t>(box) * 3 * N + (lk * B::NY + lj) * B::NX + li;
         long long v[3] = {0, 0, 0};
 #pragma unroll
         for (int d = 0; d < 3; ++d)
           if (has[d]) v[d] = at[d * N];
 #pragma unroll
         for (int d = 0; d < 3; ++d) sum[d] += ldexp(static_cast<double>(v[d]), -nbShift[nb]);
-        if (box & 1)
+        if (box < T.added)
 #pragma unroll
           for (int d = 0; d < 3; ++d)
             if (has[d]) at[d * N] = 0;
@@ -453,12 +455,12 @@ __device__ __forceinline__ void ownedNodeSums(long long* partial, const int* nbB
 // owns the closing node). ne: the components' extents.
 template <int SHAPE, class Node>
 __device__ __forceinline__ void reduceOwnedTile(const int ne[3][3], int tile, const unsigned long long* tileScan,
-                                                const int* tileShift, long long* partial, int ntx, int nty, int ntz,
+                                                const int* tileShift, const TileBoxes& T, int ntx, int nty, int ntz,
                                                 Node node) {
   constexpr int NB = 9 * (2 * Box<SHAPE>::RZ + 1);
   const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
   __shared__ int nbBox[NB], nbShift[NB];
-  coveringTiles<SHAPE>(tileScan, tileShift, tx, ty, tz, ntx, nty, ntz, nbBox, nbShift);
+  coveringTiles<SHAPE>(T, tileScan, tileShift, tx, ty, tz, ntx, nty, ntz, nbBox, nbShift);
   __syncthreads();
   const int nx = ne[0][0], ny = ne[1][1], nz = ne[2][2];  // cells
   const int i0 = tx * kTileX, wx = (tx == ntx - 1 ? nx + 1 : i0 + kTileX) - i0;
@@ -468,7 +470,7 @@ __device__ __forceinline__ void reduceOwnedTile(const int ne[3][3], int tile, co
     const int i = i0 + t % wx, j = j0 + (t / wx) % wy, k = k0 + t / (wx * wy);
     const bool has[3] = {i < nx, j < ny, k < nz};
     double sum[3];
-    ownedNodeSums<SHAPE>(partial, nbBox, nbShift, tx, ty, tz, i, j, k, has, sum);
+    ownedNodeSums<SHAPE>(T, nbBox, nbShift, tx, ty, tz, i, j, k, has, sum);
     node(i, j, k, has, sum);
   }
 }
@@ -484,14 +486,14 @@ __device__ __forceinline__ void reduceOwnedTile(const int ne[3][3], int tile, co
 // ones with integer atomics, whose sum is independent of their order.
 template <int SHAPE>
 __device__ __forceinline__ void flushRawBox(const unsigned long long* acc, const TileBox<SHAPE>& box, const int n[3][3],
-                                            long long* partial, const unsigned long long* tileScan, int tile) {
+                                            const TileBoxes& T, const unsigned long long* tileScan, int tile) {
   using B = Box<SHAPE>;
   using W = RawBox<SHAPE>;
   constexpr int N = boxNodes<SHAPE>(), NR = rawNodes<SHAPE>(), P = B::NX * B::NY, PR = W::NX * W::NY;
-  const unsigned long long tsc = tileScan[tile];
-  const bool alone = chunkField(tileScan[tile + 1]) - chunkField(tsc) == 1;
+  const int target = tileBoxOf(T, tileScan[tile], tileScan[tile + 1]);
+  const bool alone = target >= T.added;
   unsigned long long* const slot =
-      reinterpret_cast<unsigned long long*>(partial + (2 * static_cast<size_t>(occupiedField(tsc)) + !alone) * 3 * N);
+      reinterpret_cast<unsigned long long*>(T.at + static_cast<size_t>(target) * 3 * N);
   for (int t = threadIdx.x; t < 3 * P; t += blockDim.x) {
     const int d = t / P, r = t - d * P, ly = r / B::NX, lx = r - ly * B::NX;
     const int n0 = d == 0 ? n[0][0] : (d == 1 ? n[1][0] : n[2][0]);

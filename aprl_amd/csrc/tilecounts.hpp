@@ -8,7 +8,7 @@ namespace aprl_gpu {
 
 // Per-tile counts packed in one 64-bit word, so that one exclusive scan
 // over the tiles gives a tile's first chunk, its slot among the occupied
-// tiles (its fixed-point partial box) and its slot among the active tiles:
+// tiles (TileBoxes) and its slot among the active tiles:
 // chunks in bits 0-21, occupied (0 or 1) in bits 22-42, active in 43-63.
 // The fields cannot carry into each other while the totals fit them
 // (checked on the host: kMaxTiles tiles, kMaxChunks chunks).
