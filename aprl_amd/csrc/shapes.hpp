@@ -9,6 +9,7 @@
 // reference's (longitudinal_shape.h), summed in another order.
 #pragma once
 
+#include "fixedsum.hpp"
 #include "tilecounts.hpp"
 
 #include "particles.hpp"
@@ -159,19 +160,6 @@ __device__ __forceinline__ constexpr double quinticCompensation(int q) {
   return m == 0 ? -d / 64.
                 : (m == 1 ? b / 16. + 3 * d / 32.
                           : (m == 2 ? -a / 4. - b / 4. - 15 * d / 64. : 1 + a / 2. + 3 * b / 8. + 5 * d / 16.));
-}
-
-// part1 * w rounded to an integer, |part1 * w| < 2^62: two additions of
-// 1.5 2^84 and 1.5 2^52 leave the multiple of 2^32 and the rest in the low
-// words of their sums, with one rounding (an llrint of the rounded product
-// takes twice the instructions, and its product a rounding of its own).
-__device__ __forceinline__ unsigned long long fixedPoint(double part1, double w) {
-#pragma clang fp contract(off)
-  const double hi = fma(part1, w, 0x1.8p84);
-  const double lo = fma(part1, w, -(hi - 0x1.8p84)) + 0x1.8p52;
-  const unsigned long long h = static_cast<unsigned long long>(__double_as_longlong(hi));
-  const unsigned long long l = static_cast<unsigned long long>(__double_as_longlong(lo));
-  return ((h << 32) + l) - 0x4338000000000000ull;
 }
 
 // The quintic's weights along z on one segment: for t = g + hz s, s in
