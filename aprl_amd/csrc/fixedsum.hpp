@@ -19,4 +19,27 @@ __host__ __device__ __forceinline__ unsigned long long fixedPoint(double part1, 
   return ((h << 32) + l) - 0x4338000000000000ull;
 }
 
+// The quintic's compensation (quinticCompensation): numerators over
+// 1024 27 7, the weights' common denominator.
+constexpr double kQuinticDen = 193536.;
+constexpr double kQuinticNum[7] = {-1571., 17322., -95469., 352972., -95469., 17322., -1571.};
+
+// (a 2^32 + b) / kQuinticDen rounded to the nearest integer (halves up), for
+// whole a, b: the sums of kQuinticNum times the high words (|.| <= 2^30) and
+// the low words (< 2^32) of raw sums, exact in FP64 (the numerators' absolute
+// values add up to 581696 < 2^19.2). The high sum's quotient leaves a
+// remainder of at most half the denominator, which joins the low sum below
+// 2^52; that sum's quotient is off the nearest integer only where it halves.
+__host__ __device__ __forceinline__ long long quinticQuotient(double a, double b) {
+#pragma clang fp contract(off)
+  constexpr double inverse = 1.0 / kQuinticDen;
+  const double high = std::fma(a, inverse, 0x1.8p52);
+  const double left = std::fma(std::fma(-kQuinticDen, high - 0x1.8p52, a), 0x1p32, b);
+  const double low = std::fma(left, inverse, 0x1.8p52);
+  const double rest = std::fma(-kQuinticDen, low - 0x1.8p52, left);
+  const unsigned long long h = __builtin_bit_cast(unsigned long long, high);
+  const unsigned long long l = __builtin_bit_cast(unsigned long long, low);
+  return static_cast<long long>(((h << 32) + l) - 0x4338000000000000ull + (2.0 * rest >= kQuinticDen ? 1 : 0));
+}
+
 }  // namespace aprl_gpu

@@ -286,8 +286,8 @@ __global__ void __launch_bounds__(kScanThreads) kChunkList(const int* begin, con
   if (t >= ntiles) return;
   if (activeField(count)) active[activeField(sc)] = t;
   const int e = end[t];
-  int c = chunkField(sc);
-  for (int p = begin[t]; p < e; p += chunk, ++c) chunks[c] = make_int4(t, p, min(e, p + chunk), 0);
+  int c = chunkField(sc), fold = chunkField(count) > 1 ? occupiedField(sc) + 1 : 0;
+  for (int p = begin[t]; p < e; p += chunk, ++c, fold = 0) chunks[c] = make_int4(t, p, min(e, p + chunk), fold);
 }
 
 __global__ void kClearWords(unsigned* a, unsigned na, unsigned* b, unsigned nb) {
@@ -513,23 +513,27 @@ __global__ void __launch_bounds__(128) kPush(PArgs P, GArgs G, StepArgs S, unsig
 }
 
 // Deterministic tile deposition of Current::deposit (longitudinal_shape.h:
-// 175-187): one workgroup per chunk, one lane per particle, every raw tap of the chord x0 -> x1 (RawBox) accumulated into an LDS copy of the
-// tile's raw box in 64-bit fixed point; the write-out applies the shape's
-// convolution. The binary exponent comes from a bound on the whole tile's
+// 175-187): one workgroup per chunk, one lane per particle, every raw tap of
+// the chord x0 -> x1 (RawBox) accumulated into an LDS copy of the tile's raw
+// box in 64-bit fixed point; the write-out applies the shape's convolution
+// (kFoldTiles for a tile of several chunks). The binary exponent comes from a bound on the whole tile's
 // current (the shape's weight bound times the tile's particle count times
 // the largest per-particle bound the push recorded), so every chunk of a
-// tile uses the same scale. Integer addition is associative, so the LDS
-// atomics and the chunk sums are reproducible in any order; each tap is
-// rounded once, to 2^-62 of the tile bound.
+// tile uses the same scale. Integer addition is associative, so a tile's raw
+// sums are the same in any order of its entries and in any division into
+// chunks; each raw tap is rounded once, to 2^-62 of the tile bound, and a
+// node's convolved sum over the whole tile once more to that unit.
 // Bound by the LDS atomics (64 lanes on random nodes conflict) and the
 // per-particle arithmetic with two or three waves per SIMD to hide either
 // (231 registers for the quintic): 24 or 88 raw taps for a chord of two
 // segments instead of 128 or 736, added without a mask when the whole wave's
 // taps lie inside the box (fixedPoint). 64x64x512, 1e5 particles, with the
 // reference's taps, with raw taps of quadrature sums (two lanes a quintic
-// particle), and now with splineMoments: quintic 116, 60 and 36 us
-// (FP32-split 78, 44 and 35 us), binomial3-x 28, 26 and 24 us (FP32-split
-// 28, 19 and 18 us).
+// particle), and with splineMoments: quintic 116, 60 and 36 us (FP32-split 78,
+// 44 and 34 us), binomial3-x 28, 26 and 24.5 us (FP32-split 28, 19 and 17 us);
+// the chunks of larger tiles add raw sums instead of convolved ones (3993
+// nodes instead of 6171, 2541 instead of 3861) for 33 (30) and 22.5 (15.4)
+// us, and kFoldTiles.
 template <int SHAPE>
 __global__ void __launch_bounds__(kChunk) __attribute__((amdgpu_waves_per_eu(SHAPE == kShapeQuintic ? 2 : 3)))
 kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin, const int* tileEnd,
@@ -623,8 +627,39 @@ kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin,
     }
   }
   __syncthreads();
-  flushRawBox<SHAPE>(acc, box, G.ne, T, tileScan, tile);
+  flushRawBox<SHAPE>(acc, box, G.nx, G.ny, G.nz, T, tileScan, tile);
   if (err) atomicOr(errOut, err);
+}
+
+// After a deposit: the boxes of the tiles of several chunks from their raw
+// boxes. One workgroup per chunk, of which the tiles' first ones work. Bound
+// by the latency of its chain (chunk, raw box, LDS, store) in small grids:
+// 5.7 us at 64x64x512 with 1e5 particles (quintic 8.3 us), 18 us at
+// 128x128x960 with 1e6 (8.2 us with each column's loads between its stores).
+// A chunk that convolves what it adds saves this launch, but rounds each of
+// its sums, so that the current depends on the division into chunks; exact
+// (quotient and remainder added apart) it took deposit and reduction from 36
+// and 30 to 47 and 46 us (quintic, 1e5).
+template <int SHAPE>
+__global__ void __launch_bounds__(kFoldThreads) kFoldTiles(TileBoxes T, const int4* chunks, int nx, int ny, int nz,
+                                                           const unsigned* stop) {
+  const int chunk = static_cast<int>(blockIdx.x);
+  const int4 ch = chunks[chunk];
+  const unsigned stopped = stop ? *stop : 0u;
+  if (stopped || !ch.w) return;
+  foldTile<SHAPE>(chunk, ch.w - 1, tileBox<SHAPE>(ch.x, (nx + kTileX - 1) / kTileX, (ny + kTileY - 1) / kTileY), nx,
+                  ny, nz, T);
+}
+
+void foldTiles(CouplingState& C, const TileBoxes& T, const aprl_grid_geometry& g, unsigned nChunks, unsigned occupied,
+               const unsigned* stop, hipStream_t st) {
+  if (nChunks == occupied) return;  // no tile of several chunks
+  const int nx = static_cast<int>(g.nx), ny = static_cast<int>(g.ny), nz = static_cast<int>(g.nz);
+  if (C.shape == kShapeQuintic)
+    kFoldTiles<kShapeQuintic><<<nChunks, kFoldThreads, 0, st>>>(T, C.chunks.get(), nx, ny, nz, stop);
+  else
+    kFoldTiles<kShapeBinomial3X><<<nChunks, kFoldThreads, 0, st>>>(T, C.chunks.get(), nx, ny, nz, stop);
+  launchCheck("fold tiles");
 }
 
 // Node-owner reduction into J, one workgroup per active cell tile (a tile
@@ -636,21 +671,22 @@ kDeposit(PArgs P, GArgs G, StepArgs S, const int4* chunks, const int* tileBegin,
 // zero-current sums E* + E_old. J itself is only read after the last trial:
 // writeJ is off for a trial that cannot be it. Nodes of other tiles keep the
 // zeros J held at the start of the step.
-// Bound by the partials' loads (about five boxes cover a node) and, in small
-// grids, their latency: the three components' loads go together, a box that
-// the next deposit overwrites is not cleared, and J is written once a step.
-// Before and now: 19.5 -> 11.7 us (1e4 particles in 32x32x256), 34.5 -> 21 us
-// (1e5 in 64x64x512; quintic 51 -> 30 us), 213 -> 129 us (1e6 in
-// 128x128x960); FP32-split quintic, 4e6 particles, 510 and 436 -> 297 and
-// 285 us.
+// Bound by the boxes' loads (about five boxes cover a node) and, in small
+// grids, their latency: the three components' loads go together, no box is
+// cleared (the next deposit overwrites it), and J is written once a step.
+// At first, with the components one after the other and every box cleared,
+// then with the boxes of larger tiles cleared, and now: 19.5, 11.6 and 11.6 us
+// (1e4 particles in 32x32x256), 34.5, 21 and 18.5 us (1e5 in 64x64x512;
+// quintic 51, 30 and 26 us), 213, 129 and 114 us (1e6 in 128x128x960);
+// FP32-split quintic, 4e6 particles, 510 and 436, 245 and 227, 226 and 208 us.
 template <int SHAPE>
 __global__ void __launch_bounds__(256) kReduceCurrent(double* jx, double* jy, double* jz, GArgs G, const int* active,
                                                       const unsigned long long* tileScan, const int* tileShift,
-                                                      TileBoxes T, int ntx, int nty, int ntz, int writeJ) {
+                                                      const long long* boxes, int ntx, int nty, int ntz, int writeJ) {
   if (G.stop && *G.stop) return;
   const int tile = active[xcdContiguous(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   reduceOwnedTile<SHAPE>(
-      G.ne, tile, tileScan, tileShift, T, ntx, nty, ntz,
+      G.ne, tile, tileScan, tileShift, boxes, ntx, nty, ntz,
       [&](int i, int j, int k, const bool has[3], const double sum[3]) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -1013,21 +1049,23 @@ void reduceChunkStats(hipStream_t st, const double* in, int chunks, double* out)
   launchCheck("chunk stats");
 }
 
-TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, unsigned nChunks, unsigned occupied,
-                             hipStream_t st) {
-  const std::size_t extra = nChunks - occupied, added = std::min<std::size_t>(extra, occupied);
-  if (added > C.addedBoxes || occupied > C.storedBoxes) {
-    const std::size_t zeros = added > C.addedBoxes ? added + added / 2 : C.addedBoxes;
-    const std::size_t others = occupied > C.storedBoxes ? occupied + occupied / 2 : C.storedBoxes;
-    C.addedBoxes = C.storedBoxes = 0;  // none, should the allocation fail
-    C.boxes.resize(boxWords * (zeros + others));
-    if (zeros) hipCheck(hipMemsetAsync(C.boxes.get(), 0, boxWords * zeros * sizeof(long long), st), "hipMemsetAsync");
-    C.addedBoxes = zeros;
-    C.storedBoxes = others;
+TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, std::size_t rawWords, unsigned nChunks,
+                             unsigned occupied, hipStream_t st) {
+  const std::size_t extra = nChunks - occupied;
+  const std::size_t need = boxWords * occupied, raw = rawWords * std::min<std::size_t>(extra, occupied);
+  // at least 16 MiB: of 8 to 10 MB, in a process that had freed memory before,
+  // an allocation took 0.5 ms instead of 0.04 ms, a seventh of a small grid's
+  // first steps
+  if (need > C.boxes.size()) C.boxes.resize(std::max<std::size_t>(need + need / 2, 1u << 21));
+  if (raw > C.rawBoxes.size()) {
+    // at least 64 boxes, 1 to 2 MB: half of a few is soon used up
+    const std::size_t n = std::max(raw + raw / 2, 64 * rawWords);
+    C.rawBoxes.resize(n);
+    hipCheck(hipMemsetAsync(C.rawBoxes.get(), 0, n * sizeof(long long), st), "hipMemsetAsync");
   }
   const std::size_t blocks = 4 * static_cast<std::size_t>(std::max(1u, nChunks));
   if (C.reduceBlocks.size() < blocks) C.reduceBlocks.resize(blocks + blocks / 2);
-  return TileBoxes{C.boxes.get(), static_cast<int>(C.addedBoxes), extra <= occupied ? 1 : 0};
+  return TileBoxes{C.boxes.get(), C.rawBoxes.get(), extra <= occupied ? 1 : 0};
 }
 
 void reserveCouplingWords(CouplingState& C, hipStream_t st) {
@@ -1246,6 +1284,7 @@ void enqueueTrials(CouplingState& C, PlainStepContext& X, unsigned first, unsign
               A, G, S, C.chunks.get(), C.tileBegin.get(), C.tileEnd.get(), C.tileScan.get(), ntx, nty,
               X.boxes, C.tileShift.get(), errT);
         launchCheck("deposit");
+        foldTiles(C, X.boxes, F.g, nChunks, X.occupied, stop, st);
       }
       {
         ScopedKernel sk(F.profiler, st, "reduce_current");
@@ -1254,12 +1293,12 @@ void enqueueTrials(CouplingState& C, PlainStepContext& X, unsigned first, unsign
         if (quintic)
           kReduceCurrent<kShapeQuintic><<<nActive, 256, 0, st>>>(F.base(6), F.base(7), F.base(8), G,
                                                                  C.activeTiles.get(), C.tileScan.get(),
-                                                                 C.tileShift.get(), X.boxes, ntx, nty, ntz,
+                                                                 C.tileShift.get(), X.boxes.boxes, ntx, nty, ntz,
                                                                  writeJ);
         else
           kReduceCurrent<kShapeBinomial3X><<<nActive, 256, 0, st>>>(F.base(6), F.base(7), F.base(8), G,
                                                                     C.activeTiles.get(), C.tileScan.get(),
-                                                                    C.tileShift.get(), X.boxes, ntx, nty,
+                                                                    C.tileShift.get(), X.boxes.boxes, ntx, nty,
                                                                     ntz, writeJ);
         launchCheck("reduce current");
       }
@@ -1368,7 +1407,9 @@ void plainStepBegin(CouplingState& C, ParticleStore& P, const double origin[3], 
   }
   const bool quintic = C.shape == kShapeQuintic;
   const int boxN = quintic ? boxNodes<kShapeQuintic>() : boxNodes<kShapeBinomial3X>();
-  X.boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), nChunks, occupiedTiles, st);
+  const int rawN = quintic ? rawNodes<kShapeQuintic>() : rawNodes<kShapeBinomial3X>();
+  X.boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), 3 * static_cast<std::size_t>(rawN), nChunks,
+                               occupiedTiles, st);
 
   X.S = stepArgsFor(C, F.g, F.hasCpml ? &F.cpml : nullptr, F.window, origin, time, substeps);
   X.A = particleArgs(P);

@@ -184,14 +184,14 @@ struct CouplingState {
   // occupied, has an occupied neighbour; packTileCounts); the exclusive
   // scan gives the first chunk, the occupied slot and the active slot
   DeviceArray<unsigned long long> tileCounts, tileScan;
-  DeviceArray<int4> chunks;  // (tile, first particle, end particle, 0)
+  // (tile, first particle, end particle, 1 + the occupied slot of a tile of
+  // several chunks in its first one, else 0)
+  DeviceArray<int4> chunks;
   std::size_t chunkCapacity = 0;
   DeviceArray<unsigned long long> tileSums;  // of tileCounts, per workgroup of kTileCounts
   DeviceArray<unsigned> keyActive;           // live active entries per workgroup of the key kernel
-  // fixed-point current of the tiles, 3 components of an extended tile box
-  // each (TileBoxes), and the capacities of its two parts in boxes
-  DeviceArray<long long> boxes;
-  std::size_t addedBoxes = 0, storedBoxes = 0;
+  // fixed-point current of the occupied tiles (TileBoxes)
+  DeviceArray<long long> boxes, rawBoxes;
   DeviceArray<double> reduceBlocks, reduceOut;
   DeviceArray<unsigned> error;
   // cumulative boundary counters and their per-block partials
@@ -364,23 +364,27 @@ void appendParticles(ParticleStore& P, std::size_t k, const double* x3, const do
 // Error words and boundary counters of a coupling (allocated and cleared
 // once).
 void reserveCouplingWords(CouplingState& C, hipStream_t st);
-// Fixed-point current boxes of the occupied tiles, in one array: the first
-// `added` boxes are those of tiles of several chunks, which add to zeros that
-// the reduction restores; the boxes behind them, by occupied slot, are those
-// of tiles of one chunk, which stores every node. A larger tile's box is its
+// Fixed-point current of the occupied tiles, 64-bit integers scaled by
+// 2^shift (a shift per tile): an extended tile box of 3 components by
+// occupied slot, and for the tiles of several chunks a raw box, to which the
+// chunks add and which holds zeros between deposits. A tile's raw box is its
 // first chunk less its occupied slot (it advances that difference by its
 // chunks beyond the first, so the difference is its own), or its occupied
 // slot where that makes fewer boxes (byChunk = 0).
 struct TileBoxes {
-  long long* at;
-  int added, byChunk;
+  long long *boxes, *raw;
+  int byChunk;
 };
 // The step's tile boxes and residual block slots, grown with half again as
 // much headroom: a bunch that spreads over new tiles raises the need a little
 // in many steps, and every reallocation frees device memory, which waits for
-// the device. boxWords: 64-bit words of a tile's box.
-TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, unsigned nChunks, unsigned occupied,
-                             hipStream_t st);
+// the device. boxWords, rawWords: 64-bit words of a tile's boxes.
+TileBoxes reserveStepBuffers(CouplingState& C, std::size_t boxWords, std::size_t rawWords, unsigned nChunks,
+                             unsigned occupied, hipStream_t st);
+// After a deposit: the boxes of the tiles of several chunks from their raw
+// boxes (foldTile); a non-null stop word that is set skips it.
+void foldTiles(CouplingState& C, const TileBoxes& T, const aprl_grid_geometry& g, unsigned nChunks, unsigned occupied,
+               const unsigned* stop, hipStream_t st);
 // Boundary-event commit after the converged trial: entry states and
 // weights, removed-entry count and the counters, skipped on the device when
 // the trial's error word carries no kEvtAny. R is the store's real type.

@@ -521,11 +521,11 @@ kDepositSplit(PArgs32 P, GArgs32 G, StepArgs S, const int4* chunks, const int* t
     if (p0 < ch.z) particle(p0);
   }
   __syncthreads();
-  flushRawBox<SHAPE>(acc, box, G.ne, T, tileScan, tile);
+  flushRawBox<SHAPE>(acc, box, G.nx, G.ny, G.nz, T, tileScan, tile);
   if (err) atomicOr(errOut, err);
 }
 
-// Node-owner reduction of the tile partials (sums in FP64): with J the FP32
+// Node-owner reduction of the tile boxes (sums in FP64): with J the FP32
 // current, rounded once (only the last trial's is read), with ESUM the
 // trial's E_cand + E_old (applyCurrentSource(-1) on the preview,
 // source_coupling.cpp:84-89) for the next residual gather, from the
@@ -533,11 +533,11 @@ kDepositSplit(PArgs32 P, GArgs32 G, StepArgs S, const int4* chunks, const int* t
 template <int SHAPE, bool J, bool ESUM>
 __global__ void __launch_bounds__(256) kReduceCurrentSplit(float* jx, float* jy, float* jz, GArgs32 G,
                                                            const int* active, const unsigned long long* tileScan,
-                                                           const int* tileShift, TileBoxes T, int ntx,
+                                                           const int* tileShift, const long long* boxes, int ntx,
                                                            int nty, int ntz) {
   const int tile = active[xcdContiguous(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x))];
   reduceOwnedTile<SHAPE>(
-      G.ne, tile, tileScan, tileShift, T, ntx, nty, ntz,
+      G.ne, tile, tileScan, tileShift, boxes, ntx, nty, ntz,
       [&](int i, int j, int k, const bool has[3], const double sum[3]) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -782,14 +782,14 @@ PArgs32 particleArgs32(SplitStore& P, const FieldState32& F) {
 
 // Entries per chunk: kChunk, and up to 8 times as many from 2^19 entries on,
 // where a chunk's fixed cost (staging its tile's fields; clearing its tile's
-// current and writing it out, for the quintic 6171 atomics unless the tile
-// has one chunk) is then paid for several entries a lane. At least 1024
+// current and writing it out, for the quintic up to 3993 atomics unless the
+// tile has one chunk) is then paid for several entries a lane. At least 1024
 // full chunks remain, four for each CU.
-// At 4e6 entries in 128x128x960 (quintic): deposit 658 -> 536 us, current
-// reduction 297 and 285 -> 245 and 228 us (fewer tiles of several chunks),
-// gathers 331 -> 316 us (with B staged, sampleQuinticB); at 6e5 in 64x64x512
-// 565 -> 533 us a binomial3-x step, 733 -> 704 us a quintic one. The FP64
-// kernels keep one entry per lane: their loop takes 54 more registers and at 1e6 entries the step was 1% slower with it.
+// At 4e6 entries in 128x128x960 (quintic): deposit 658 -> 536 us (527 us with
+// raw sums added), gathers 331 -> 316 us (with B staged, sampleQuinticB); at
+// 6e5 in 64x64x512 565 -> 533 us a binomial3-x step, 733 -> 704 us a quintic
+// one. The FP64 kernels keep one entry per lane: their loop takes 54 more
+// registers and at 1e6 entries the step was 1% slower with it.
 int chunkSize32(int n) {
   int size = kChunk;
   for (int m = n >> 18; m > 1 && size < 8 * kChunk; m >>= 1) size *= 2;
@@ -1026,7 +1026,9 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
   }
   const bool quintic = C.shape == kShapeQuintic;
   const int boxN = quintic ? boxNodes<kShapeQuintic>() : boxNodes<kShapeBinomial3X>();
-  const TileBoxes boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), nChunks, occupiedTiles, st);
+  const int rawN = quintic ? rawNodes<kShapeQuintic>() : rawNodes<kShapeBinomial3X>();
+  const TileBoxes boxes = reserveStepBuffers(C, 3 * static_cast<std::size_t>(boxN), 3 * static_cast<std::size_t>(rawN),
+                                             nChunks, occupiedTiles, st);
 
   const StepArgs& S = X.S;
   PArgs32 A = particleArgs32(P, F);
@@ -1076,6 +1078,7 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
       }
 #undef APRL_DEPOSIT32
       launchCheck("deposit");
+      foldTiles(C, boxes, F.g, nChunks, occupiedTiles, nullptr, st);
     }
     // the last trial's E_cand + E_old is read only by a verifying residual
     const bool esum = !last || verify;
@@ -1085,7 +1088,7 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
       const bool writeJ = last || C.refCurrent;
 #define APRL_REDUCE32(SH, WJ, WE)                                                                                     \
   kReduceCurrentSplit<SH, WJ, WE><<<nActive, 256, 0, st>>>(j[0], j[1], j[2], G, C.activeTiles.get(), C.tileScan.get(), \
-                                                           C.tileShift.get(), boxes, ntx, nty, ntz)
+                                                           C.tileShift.get(), boxes.boxes, ntx, nty, ntz)
       if (quintic) {
         if (writeJ && esum) APRL_REDUCE32(kShapeQuintic, true, true);
         else if (writeJ) APRL_REDUCE32(kShapeQuintic, true, false);

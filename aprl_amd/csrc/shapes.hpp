@@ -363,25 +363,19 @@ __device__ __forceinline__ unsigned rawDepositMask(const TileBox<SHAPE>& box, co
   return mask;
 }
 
-// Fixed-point tile boxes (TileBoxes): 3 components x boxNodes<SHAPE>() 64-bit
-// integers scaled by 2^shift (shift per tile). A tile's box from its scanned
-// counts; -1 for an unoccupied tile.
-__device__ __forceinline__ int tileBoxOf(const TileBoxes& T, unsigned long long scan, unsigned long long next) {
-  const int chunks = chunkField(next) - chunkField(scan);
-  if (chunks <= 0) return -1;
-  const int slot = occupiedField(scan);
-  if (chunks == 1) return T.added + slot;
-  return T.byChunk ? chunkField(scan) - slot : slot;
+// The raw box of a tile of several chunks (TileBoxes).
+template <int SHAPE>
+__device__ __forceinline__ long long* rawBoxOf(const TileBoxes& T, int firstChunk, int slot) {
+  return T.raw + static_cast<size_t>(T.byChunk ? firstChunk - slot : slot) * 3 * rawNodes<SHAPE>();
 }
 
 // The owner side's table of the covering tiles of tile (tx, ty, tz): threads
 // 0..9(2RZ+1)-1 fill, per neighbour offset (oz + RZ, oy + 1, ox + 1), the
-// box (tileBoxOf) and the exponent from the tile scan. The caller
-// synchronizes before reading it.
+// box (its occupied slot; -1: unoccupied) and the exponent from the tile
+// scan. The caller synchronizes before reading it.
 template <int SHAPE>
-__device__ __forceinline__ void coveringTiles(const TileBoxes& T, const unsigned long long* tileScan,
-                                              const int* tileShift, int tx, int ty, int tz, int ntx, int nty, int ntz,
-                                              int* nbBox, int* nbShift) {
+__device__ __forceinline__ void coveringTiles(const unsigned long long* tileScan, const int* tileShift, int tx,
+                                              int ty, int tz, int ntx, int nty, int ntz, int* nbBox, int* nbShift) {
   constexpr int RZ = Box<SHAPE>::RZ, NB = 9 * (2 * RZ + 1);
   if (threadIdx.x >= NB) return;
   const int nb = static_cast<int>(threadIdx.x);
@@ -389,8 +383,11 @@ __device__ __forceinline__ void coveringTiles(const TileBoxes& T, const unsigned
   int box = -1, sh = 0;
   if (x >= 0 && x < ntx && y >= 0 && y < nty && z >= 0 && z < ntz) {
     const int s = (z * nty + y) * ntx + x;
-    box = tileBoxOf(T, tileScan[s], tileScan[s + 1]);
-    if (box >= 0) sh = tileShift[s];
+    const unsigned long long sc = tileScan[s];
+    if (chunkField(tileScan[s + 1]) > chunkField(sc)) {
+      box = occupiedField(sc);
+      sh = tileShift[s];
+    }
   }
   nbBox[nb] = box;
   nbShift[nb] = sh;
@@ -400,11 +397,10 @@ __device__ __forceinline__ void coveringTiles(const TileBoxes& T, const unsigned
 // components' three values together (their addresses differ by a constant,
 // and three loads are in flight per covering tile): over the neighbour tiles
 // whose extended box covers the node, in ascending (z, y, x) tile order, the
-// partials converted with that tile's exponent; entries of a larger tile's
-// box are cleared for the next deposit. has: whether the component owns the
-// node.
+// tiles' sums converted with that tile's exponent. has: whether the component
+// owns the node.
 template <int SHAPE>
-__device__ __forceinline__ void ownedNodeSums(const TileBoxes& T, const int* nbBox, const int* nbShift, int tx, int ty,
+__device__ __forceinline__ void ownedNodeSums(const long long* boxes, const int* nbBox, const int* nbShift, int tx, int ty,
                                               int tz, int i, int j, int k, const bool has[3], double sum[3]) {
   using B = Box<SHAPE>;
   constexpr int N = boxNodes<SHAPE>(), RZ = B::RZ;
@@ -424,17 +420,13 @@ __device__ __forceinline__ void ownedNodeSums(const TileBoxes& T, const int* nbB
         const int box = nbBox[nb];
         if (box < 0) continue;
         const int li = i - (x * kTileX - B::X0), lj = j - (y * kTileY - B::Y0), lk = k - (z * kTileZ - B::Z0);
-        long long* const at = T.at + static_cast<size_t>(box) * 3 * N + (lk * B::NY + lj) * B::NX + li;
+        const long long* const at = boxes + static_cast<size_t>(box) * 3 * N + (lk * B::NY + lj) * B::NX + li;
         long long v[3] = {0, 0, 0};
 #pragma unroll
         for (int d = 0; d < 3; ++d)
           if (has[d]) v[d] = at[d * N];
 #pragma unroll
         for (int d = 0; d < 3; ++d) sum[d] += ldexp(static_cast<double>(v[d]), -nbShift[nb]);
-        if (box < T.added)
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-            if (has[d]) at[d * N] = 0;
       }
 }
 
@@ -443,12 +435,12 @@ __device__ __forceinline__ void ownedNodeSums(const TileBoxes& T, const int* nbB
 // owns the closing node). ne: the components' extents.
 template <int SHAPE, class Node>
 __device__ __forceinline__ void reduceOwnedTile(const int ne[3][3], int tile, const unsigned long long* tileScan,
-                                                const int* tileShift, const TileBoxes& T, int ntx, int nty, int ntz,
+                                                const int* tileShift, const long long* boxes, int ntx, int nty, int ntz,
                                                 Node node) {
   constexpr int NB = 9 * (2 * Box<SHAPE>::RZ + 1);
   const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
   __shared__ int nbBox[NB], nbShift[NB];
-  coveringTiles<SHAPE>(T, tileScan, tileShift, tx, ty, tz, ntx, nty, ntz, nbBox, nbShift);
+  coveringTiles<SHAPE>(tileScan, tileShift, tx, ty, tz, ntx, nty, ntz, nbBox, nbShift);
   __syncthreads();
   const int nx = ne[0][0], ny = ne[1][1], nz = ne[2][2];  // cells
   const int i0 = tx * kTileX, wx = (tx == ntx - 1 ? nx + 1 : i0 + kTileX) - i0;
@@ -458,44 +450,33 @@ __device__ __forceinline__ void reduceOwnedTile(const int ne[3][3], int tile, co
     const int i = i0 + t % wx, j = j0 + (t / wx) % wy, k = k0 + t / (wx * wy);
     const bool has[3] = {i < nx, j < ny, k < nz};
     double sum[3];
-    ownedNodeSums<SHAPE>(T, nbBox, nbShift, tx, ty, tz, i, j, k, has, sum);
+    ownedNodeSums<SHAPE>(boxes, nbBox, nbShift, tx, ty, tz, i, j, k, has, sum);
     node(i, j, k, has, sum);
   }
 }
 
-// The deposit side's write-out of one chunk's LDS raw box acc (3
-// components): the shape's convolution is applied on the way out, one thread
-// per (x, y) column of the box, in integers for binomial3-x (weights 1, 2, 1
-// twice, then a division by 16; the sums are kept as 16 h + l, so that
-// nothing is lost before it) and in FP64 for the quintic's compensation; each
-// result is rounded once to the fixed-point unit, as a tap is. Nodes outside
-// a component (n: the components' extents) get nothing. A tile of one chunk
-// stores every node of its box; chunks of a larger tile add their nonzero
-// ones with integer atomics, whose sum is independent of their order.
+// A tile's box from its raw box (3 components each): the shape's convolution,
+// one thread per (x, y) column of the box, each node's exact sum rounded once
+// to the fixed-point unit. Binomial3-x (weights 1, 2, 1 twice, then a division
+// by 16) keeps its sums as 16 h + l; the quintic sums whole numbers in FP64, a
+// raw sum's high and low words apart (quinticQuotient). Nodes outside a
+// component (of nx x ny x nz cells) are not written; none of them is read.
 template <int SHAPE>
-__device__ __forceinline__ void flushRawBox(const unsigned long long* acc, const TileBox<SHAPE>& box, const int n[3][3],
-                                            const TileBoxes& T, const unsigned long long* tileScan, int tile) {
+__device__ __forceinline__ void convolveRawBox(const long long* raw, const TileBox<SHAPE>& box, int nx, int ny, int nz,
+                                               long long* slot) {
   using B = Box<SHAPE>;
   using W = RawBox<SHAPE>;
   constexpr int N = boxNodes<SHAPE>(), NR = rawNodes<SHAPE>(), P = B::NX * B::NY, PR = W::NX * W::NY;
-  const int target = tileBoxOf(T, tileScan[tile], tileScan[tile + 1]);
-  const bool alone = target >= T.added;
-  unsigned long long* const slot =
-      reinterpret_cast<unsigned long long*>(T.at + static_cast<size_t>(target) * 3 * N);
   for (int t = threadIdx.x; t < 3 * P; t += blockDim.x) {
     const int d = t / P, r = t - d * P, ly = r / B::NX, lx = r - ly * B::NX;
-    const int n0 = d == 0 ? n[0][0] : (d == 1 ? n[1][0] : n[2][0]);
-    const int n1 = d == 0 ? n[0][1] : (d == 1 ? n[1][1] : n[2][1]);
-    const int n2 = d == 0 ? n[0][2] : (d == 1 ? n[1][2] : n[2][2]);
+    const int n0 = nx + (d != 0), n1 = ny + (d != 1), n2 = nz + (d != 2);
     const int i = box.x0 + lx, j = box.y0 + ly;
     if (i < 0 || i >= n0 || j < 0 || j >= n1) continue;
-    unsigned long long* const out = slot + d * N + ly * B::NX + lx;
-    const long long* const in = reinterpret_cast<const long long*>(acc) + d * NR + ly * W::NX;
+    long long* const out = slot + d * N + ly * B::NX + lx;
+    const long long* const in = raw + d * NR + ly * W::NX;
     auto put = [&](int lk, long long val) {
       const int k = box.z0 + lk;
-      if (k < 0 || k >= n2) return;
-      if (alone) out[lk * P] = static_cast<unsigned long long>(val);
-      else if (val) atomicAdd(out + lk * P, static_cast<unsigned long long>(val));
+      if (k >= 0 && k < n2) out[lk * P] = val;
     };
     if constexpr (SHAPE == kShapeBinomial3X) {
       long long h0 = 0, h1 = 0;  // the two planes before, summed in x
@@ -518,19 +499,75 @@ __device__ __forceinline__ void flushRawBox(const unsigned long long* acc, const
         l1 = l2;
       }
     } else {
-      double raw[W::NZ];
+      double high[W::NZ], low[W::NZ];
 #pragma unroll
-      for (int m = 0; m < W::NZ; ++m) raw[m] = static_cast<double>(in[m * PR + lx]);
+      for (int m = 0; m < W::NZ; ++m) {
+        const long long v = in[m * PR + lx];
+        high[m] = static_cast<double>(static_cast<int>(v >> 32));
+        low[m] = static_cast<double>(static_cast<unsigned>(v));
+      }
 #pragma unroll
       for (int lk = 0; lk < B::NZ; ++lk) {
-        double sum = 0.0;
+        double a = 0.0, b = 0.0;
 #pragma unroll
         for (int q = 0; q < 7; ++q)
-          if (lk - q >= 0 && lk - q < W::NZ) sum += quinticCompensation(q) * raw[lk - q];
-        put(lk, llrint(sum));
+          if (lk - q >= 0 && lk - q < W::NZ) {
+            a = fma(kQuinticNum[q], high[lk - q], a);
+            b = fma(kQuinticNum[q], low[lk - q], b);
+          }
+        put(lk, quinticQuotient(a, b));
       }
     }
   }
+}
+
+// The deposit side's write-out of one chunk's LDS raw box acc (3
+// components). A tile of one chunk writes its box; chunks of a larger tile
+// add their nonzero raw sums to the tile's raw box with integer atomics,
+// whose sums do not depend on their order or on how the tile's entries fall
+// into chunks, for foldTile to write the box from.
+template <int SHAPE>
+__device__ __forceinline__ void flushRawBox(const unsigned long long* acc, const TileBox<SHAPE>& box, int nx, int ny,
+                                            int nz, const TileBoxes& T, const unsigned long long* tileScan, int tile) {
+  const unsigned long long sc = tileScan[tile];
+  if (chunkField(tileScan[tile + 1]) - chunkField(sc) == 1) {
+    convolveRawBox<SHAPE>(reinterpret_cast<const long long*>(acc), box, nx, ny, nz,
+                          T.boxes + static_cast<size_t>(occupiedField(sc)) * 3 * boxNodes<SHAPE>());
+    return;
+  }
+  unsigned long long* const raw = reinterpret_cast<unsigned long long*>(rawBoxOf<SHAPE>(T, chunkField(sc), occupiedField(sc)));
+  for (int t = threadIdx.x; t < 3 * rawNodes<SHAPE>(); t += blockDim.x) {
+    const unsigned long long val = acc[t];
+    if (val) atomicAdd(raw + t, val);
+  }
+}
+
+// A thread takes one column of a box (429 or 363).
+constexpr int kFoldThreads = 512;
+// The box of a tile of several chunks (its first chunk, its occupied slot)
+// from its raw box, which is cleared for the next deposit.
+template <int SHAPE>
+__device__ __forceinline__ void foldTile(int firstChunk, int slot, const TileBox<SHAPE>& box, int nx, int ny, int nz,
+                                         const TileBoxes& T) {
+  constexpr int N = 3 * rawNodes<SHAPE>(), kPer = (N + kFoldThreads - 1) / kFoldThreads;
+  __shared__ long long sums[N];
+  long long* const raw = rawBoxOf<SHAPE>(T, firstChunk, slot);
+  long long v[kPer];  // every load ahead of the first store
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const int t = static_cast<int>(threadIdx.x) + r * kFoldThreads;
+    v[r] = t < N ? raw[t] : 0;
+  }
+#pragma unroll
+  for (int r = 0; r < kPer; ++r) {
+    const int t = static_cast<int>(threadIdx.x) + r * kFoldThreads;
+    if (t < N) {
+      sums[t] = v[r];
+      raw[t] = 0;
+    }
+  }
+  __syncthreads();
+  convolveRawBox<SHAPE>(sums, box, nx, ny, nz, T.boxes + static_cast<size_t>(slot) * 3 * boxNodes<SHAPE>());
 }
 
 // The value one lane below (kRowBelow) or above (kRowAbove) in a row of 16

@@ -1,6 +1,7 @@
 """The deposit's fixed-point arithmetic (aprl_amd/csrc/fixedsum.hpp), compiled
 for the host and compared with 128-bit integers (tests/cpp/fixedsum_check.cpp):
-a tap is its product rounded once."""
+a tap is its product rounded once, and the quintic's weights applied to raw
+sums lose nothing."""
 import os
 import subprocess
 
