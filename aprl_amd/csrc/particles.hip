@@ -4,9 +4,11 @@
 // current, residual gathers with fixed-order reductions, and the Picard
 // orchestration.
 //
-// Per-particle arithmetic follows source_coupling_math.h / source_coupling.cpp
-// / longitudinal_shape.h in the reference's association order (contraction
-// off), so with identical field inputs a push is bitwise the reference's.
+// The push follows source_coupling_math.h / source_coupling.cpp in the
+// reference's association order (contraction off), so with identical field
+// inputs it is bitwise the reference's. The gathers' and the deposit's weights
+// are longitudinal_shape.h's summed in another order, with contraction
+// (shapes.hpp).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -31,7 +33,6 @@ struct GArgs {
   int nx, ny, nz;          // cells
   double o[3], h[3];
   double negS;             // (-1*dt)/eps0, applyCurrentSource(-1)
-  int smoothX;
   // the Picard stop word: a trial's kernels return at once when it is set
   // (null for work that always runs)
   const unsigned* stop;
@@ -53,8 +54,7 @@ struct PArgs {
   double* wend;      // carrier end weight
   const double* w;   // weight slot (a carrier's current weight)
   const double* beta;  // held speed of held entries
-  const unsigned* tileOf;         // sorted tile key of each entry
-  unsigned long long* tileBound;  // per tile: largest particle current bound
+  const unsigned long long* tileBound;  // per tile: largest entry current bound
   double scaleDen;   // dx*dy*dz*dt
   int n;
 };
@@ -518,7 +518,7 @@ __global__ void __launch_bounds__(128) kPush(PArgs P, GArgs G, StepArgs S, unsig
 // box in 64-bit fixed point; the write-out applies the shape's convolution
 // (kFoldTiles for a tile of several chunks). The binary exponent comes from a bound on the whole tile's
 // current (the shape's weight bound times the tile's particle count times
-// the largest per-particle bound the push recorded), so every chunk of a
+// the largest bound of one entry, set by the sort), so every chunk of a
 // tile uses the same scale. Integer addition is associative, so a tile's raw
 // sums are the same in any order of its entries and in any division into
 // chunks; each raw tap is rounded once, to 2^-62 of the tile bound, and a
@@ -728,7 +728,6 @@ static GArgs gatherArgs(const CouplingState& C, const FieldState& F, const doubl
   G.nz = static_cast<int>(F.g.nz);
   G.h[0] = F.g.dx; G.h[1] = F.g.dy; G.h[2] = F.g.dz;
   G.negS = -1.0 * F.g.dt / kEps0;
-  G.smoothX = C.smoothX ? 1 : 0;
   return G;
 }
 
@@ -1414,7 +1413,6 @@ void plainStepBegin(CouplingState& C, ParticleStore& P, const double origin[3], 
   X.S = stepArgsFor(C, F.g, F.hasCpml ? &F.cpml : nullptr, F.window, origin, time, substeps);
   X.A = particleArgs(P);
   X.A.scaleDen = F.g.dx * F.g.dy * F.g.dz * F.g.dt;
-  X.A.tileOf = P.keySorted.get();
   X.A.tileBound = C.tileBound.get();
   X.G = gatherArgs(C, F, origin);
   X.G.stop = C.error.get() + kStopWord;

@@ -176,9 +176,9 @@ struct CouplingState {
   // tiles: particle range, fixed-point exponent of the tile's current,
   // active-tile list
   DeviceArray<int> tileBegin, tileEnd, tileShift, activeTiles;
-  // per tile: the largest current bound of one of its particles in the
-  // trial (bit pattern of a non-negative double; written by the push,
-  // read by the deposit, cleared by the current reduction and the sort)
+  // per tile: the largest current bound of one of its entries in the step
+  // (bit pattern of a non-negative double; cleared by the sort's key kernel,
+  // raised by its permute, read by the deposit)
   DeviceArray<unsigned long long> tileBound;
   // per tile (+1 entry for the scan totals): packed counts (chunks,
   // occupied, has an occupied neighbour; packTileCounts); the exclusive

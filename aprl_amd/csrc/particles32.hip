@@ -5,9 +5,10 @@
 // The step is the FP64 form's (tile sort, orbit gathers from LDS-staged
 // tile boxes, Lapenta-Markidis push, fixed-point tile deposition, owner
 // reduction) with these differences:
-//  * shape weights, chord cuts and gathers run in FP32 on coordinates taken
-//    relative to the particle's start cell, so the in-cell offset keeps its
-//    24 bits whatever the absolute position;
+//  * chord cuts, binomial3-x weights and gathers run in FP32 on coordinates
+//    taken relative to the particle's start cell, so the in-cell offset keeps
+//    its 24 bits whatever the absolute position; the quintic's weights are
+//    formed in FP64 from those coordinates (rawSegment);
 //  * the push converts its inputs to FP64 and reuses the FP64 orbit push
 //    (prescribed magnets, Newton root, boundary checks) on absolute box
 //    coordinates, then stores the end point as cell + FP32 offset again;
@@ -38,7 +39,6 @@ struct GArgs32 {
   int oc[3];       // absolute lattice cell of the grid origin
   float ch[3];     // c dt / h per axis (ballistic guess, cells per unit u/gamma)
   float negS;      // (-1*dt)/eps0
-  int smoothX;
 };
 
 struct PArgs32 {
@@ -60,8 +60,7 @@ struct PArgs32 {
   float* wend;       // carrier end weight
   const float* w;    // weight slot (a carrier's current weight)
   const float* beta; // held speed of held entries
-  const unsigned* tileOf;         // sorted tile key of each entry
-  unsigned long long* tileBound;  // per tile: largest particle current bound
+  const unsigned long long* tileBound;  // per tile: largest entry current bound
   float kq[3];  // h_a / (dx dy dz dt): current density per unit charge and cell of motion
   double h[3];
   int n;
@@ -126,12 +125,9 @@ __device__ bool clipChord(const GArgs32& G, Chord32& c, float& kept, unsigned& e
 }
 
 // ---------------------------------------------------------------------------
-// Gathers from the staged tile box.
+// Sort.
 
 __device__ __forceinline__ int clampIndex32(int v, int n) { return v < 0 ? 0 : (v > n - 1 ? n - 1 : v); }
-
-// ---------------------------------------------------------------------------
-// Sort.
 
 __global__ void kTileKeys32(const int* cx, const int* cy, const int* cz, const float* oz, int* state, int n,
                             GArgs32 G, int ntx, int nty, unsigned* key, TileRangeArgs R, SortArgs K, DigitCounts D,
@@ -349,10 +345,7 @@ __global__ void __launch_bounds__(kChunk) kGatherChunks32(PArgs32 P, GArgs32 G, 
   if (err) atomicOr(errOut, err);
 }
 
-// One entry of kPushSplit; returns the entry's current bound: the largest
-// |scale_a| of its FP32 chord as the deposit forms it (q kq_a v_a), plus,
-// for a held entry whose release kink splits the path, the held leg's
-// largest scale.
+// One entry of kPushSplit.
 __device__ __forceinline__ void pushSplitEntry(const PArgs32& P, const StepArgs& S, double o0, double o1, double o2,
                                                int p, unsigned* errOut) {
   unsigned err = 0;
@@ -404,7 +397,7 @@ __device__ __forceinline__ void pushSplitEntry(const PArgs32& P, const StepArgs&
 // push on absolute box coordinates (origin o = the grid origin cell times
 // h) or a carrier's straight move (position += dt u c / gamma), the
 // segment's boundary events, and the end point split again into cell +
-// FP32 offset; then the entries' tile current bounds.
+// FP32 offset.
 __global__ void __launch_bounds__(128) kPushSplit(PArgs32 P, StepArgs S, double o0, double o1, double o2,
                                                   unsigned* errOut) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
@@ -742,7 +735,6 @@ GArgs32 gatherArgs32(CouplingState& C, const FieldState32& F, const int oc[3]) {
   G.ch[1] = static_cast<float>(F.g.dt * kC / F.g.dy);
   G.ch[2] = static_cast<float>(F.g.dt * kC / F.g.dz);
   G.negS = static_cast<float>(-1.0 * F.g.dt / kEps0);
-  G.smoothX = C.smoothX ? 1 : 0;
   return G;
 }
 
@@ -1032,7 +1024,6 @@ void splitStepMiddle(CouplingState& C, SplitStore& P) {
 
   const StepArgs& S = X.S;
   PArgs32 A = particleArgs32(P, F);
-  A.tileOf = P.keySorted.get();
   A.tileBound = C.tileBound.get();
   const bool verify = C.splitVerify;
   const bool loop = chunkSize32(X.sortedEntries) > kChunk;

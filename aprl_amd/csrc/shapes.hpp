@@ -98,25 +98,6 @@ struct TileBox {
     using W = RawBox<SHAPE>;
     return ((k - (z0 + W::HZ)) * W::NY + (j - y0)) * W::NX + (i - (x0 + W::HX));
   }
-  __device__ int local(int i, int j, int k, unsigned& err) const {
-    const unsigned li = static_cast<unsigned>(i - x0), lj = static_cast<unsigned>(j - y0),
-                   lk = static_cast<unsigned>(k - z0);
-    if (li >= static_cast<unsigned>(Box<SHAPE>::NX) || lj >= static_cast<unsigned>(Box<SHAPE>::NY) ||
-        lk >= static_cast<unsigned>(Box<SHAPE>::NZ)) {
-      err |= kErrTileHalo;
-      return -1;
-    }
-    return static_cast<int>((lk * Box<SHAPE>::NY + lj) * Box<SHAPE>::NX + li);
-  }
-  // box contains [i, i + wx) x [j, j + wy) x [k, k + wz)
-  __device__ bool holds(long long i, long long j, long long k, int wx, int wy, int wz) const {
-    return i >= x0 && i + wx <= x0 + Box<SHAPE>::NX && j >= y0 && j + wy <= y0 + Box<SHAPE>::NY && k >= z0 &&
-           k + wz <= z0 + Box<SHAPE>::NZ;
-  }
-  __device__ int base(long long i, long long j, long long k) const {
-    return (static_cast<int>(k - z0) * Box<SHAPE>::NY + static_cast<int>(j - y0)) * Box<SHAPE>::NX +
-           static_cast<int>(i - x0);
-  }
 };
 template <int SHAPE>
 __device__ __forceinline__ TileBox<SHAPE> tileBox(int tile, int ntx, int nty) {

@@ -51,8 +51,8 @@ def kernel_bytes(w, name, tiles, chunks, active=0):
     plus 2 words per active CPML history entry; the zero-current preview
     9 words per node of each active 8x8x4 tile (read 3 B, 3 E; write E* +
     E_old). Particles: push 14 words/particle (read x, u, q, m, 6
-    fields; write x, u); gathers 14 words/particle plus 9 words per cell of
-    each occupied 8x8x4 tile (E*, E_old, B); deposit 7 words/particle (x0,
+    fields; write x, u); gathers 14 words/particle plus 6 words per cell of
+    each occupied 8x8x4 tile (E* + E_old or E_cand + E_old, B); deposit 7 words/particle (x0,
     x1, q) plus 3 words per node of each occupied tile's 13x11x9 extended
     box."""
     cells = w.cells
@@ -71,7 +71,7 @@ def kernel_bytes(w, name, tiles, chunks, active=0):
     if name == "push":
         return WORD * 14 * n
     if name in ("gather", "residual"):
-        return WORD * (14 * n + 9 * tile_cells * tiles)
+        return WORD * (14 * n + 6 * tile_cells * tiles)
     if name == "deposit":
         return WORD * (7 * n + 3 * ext_nodes * tiles)
     return None
