@@ -4,6 +4,8 @@ every inner tile holds one entry; the growth of the memory in use over the
 step against one box per occupied tile (with the headroom of half) and the
 step's other buffers, in the driver's granularity of 2 MiB each.
 """
+import gc
+
 import numpy as np
 import pytest
 import torch
@@ -35,6 +37,7 @@ def test_first_step_memory(shape, precision):
     win.beginStep(0, 50)
     gpu.advanceMagnetic()
     win.setInlet()
+    gc.collect()  # stores and grids of other tests, if any are left
     torch.cuda.synchronize()
     before = torch.cuda.mem_get_info()[0]
     cg.step(store, np.zeros(3), 0.0)
