@@ -2,7 +2,7 @@
 one chunk needs one box, whatever the number of occupied tiles. A window whose
 every inner tile holds one entry; the growth of the memory in use over the
 step against one box per occupied tile (with the headroom of half) and the
-step's other buffers, in the driver's granularity of 2 MiB each.
+step's other buffers, 2 MiB granules each.
 """
 import gc
 
